@@ -254,7 +254,8 @@ int qwen_spec_accept(const int64_t* nxt, const int64_t* tok, int64_t* hist, int3
  * epilogue epi = 0 store (bf16(acc)), 1 residual add (out = bf16(residual + bf16(acc));
  * residual may alias out), 2 SwiGLU (pair-interleaved gate|up weight of N = 2I rows; out has
  * I columns: bf16(bf16(silu(bf16(g))) * bf16(u))). x: [M, K] row-major with M * K < 2^31;
- * N % 128 == 0, K % 64 == 0; out / residual: [M, ld_out], ld_out % 8 == 0.
+ * N % 128 == 0, K % 64 == 0; out / residual: [M, ld_out], ld_out % 8 == 0. Any bf16 element may be
+ * the first of x, w_tiled, out and residual; x and w_tiled on 16-byte boundaries are the fast case.
  * Replaces the prompt forward's projections, engine/engine.py:1191-1221 (_mm / cuBLAS on
  * B*S rows) with the fused epilogues of engine/kernels/gemm_fused.py:136-173. */
 int qwen_gemm(const void* x, const void* w_tiled, void* out, int M, int N, int K, int ld_out, const void* residual,

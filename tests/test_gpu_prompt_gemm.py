@@ -83,3 +83,38 @@ def test_output_at_8_byte_alignment(qops, M, kind):
         out.copy_(res)
     got = qops.gemm(x, t, residual=out if kind == "res" else None, silu_pair=kind == "silu", out=out)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("which,off", [("x", 1), ("x", 2), ("x", 4), ("w", 1), ("w", 4), ("xw", 5)])
+@pytest.mark.parametrize("kind,N,K,M", [("plain", 384, 640, 5), ("res", 512, 192, 129), ("silu", 640, 128, 300),
+                                        ("plain", 128, 64, 1), ("res", 128, 64, 257), ("silu", 256, 1088, 64),
+                                        ("plain", 6144, 128, 1100), ("silu", 6144, 448, 700),
+                                        ("res", 6144, 320, 2200)])
+def test_operands_off_a_16_byte_boundary(qops, which, off, kind, N, K, M):
+    """Rows and weights that start at any bf16 element, with fewer k stages than LDS slots and more, in both tiles
+    (the large one past 256 small ones: N = 6144), and with several tiles of a workgroup (2,200 rows): the same bits
+    as from aligned operands."""
+    from qwen_hip import _lib
+    x, w, res = _inputs(N, K, M, seed=M + off)
+    t = qops.tile_weight(w, pair=kind == "silu")
+
+    def shifted(v):
+        flat = torch.empty(v.numel() + off, dtype=BF16, device=DEV)[off:]
+        assert flat.data_ptr() % 16 == 2 * off
+        return flat.view(v.shape).copy_(v)
+
+    def entry(x, t):   # without ops.gemm's aligned copy of x
+        out = torch.empty((M, N // 2 if kind == "silu" else N), dtype=BF16, device=DEV)
+        _lib.call("qwen_gemm", x.data_ptr(), t.data.data_ptr(), out.data_ptr(), M, N, K, out.shape[1],
+                  res.data_ptr() if kind == "res" else None, {"plain": 0, "res": 1, "silu": 2}[kind],
+                  torch.cuda.current_stream().cuda_stream)
+        return out
+
+    def call(x, t):
+        return qops.gemm(x, t, residual=res if kind == "res" else None, silu_pair=kind == "silu")
+
+    want = call(x, t)
+    ts = qops.TiledWeight(shifted(t.data), N, K, t.pair) if "w" in which else t
+    xs = shifted(x) if "x" in which else x
+    assert torch.equal(entry(xs, ts), want)
+    assert torch.equal(call(xs, ts), want)

@@ -32,6 +32,7 @@ namespace {
 enum { PEPI_STORE = 0, PEPI_RES = 1, PEPI_SWIGLU = 2 };
 
 typedef unsigned pv4 __attribute__((ext_vector_type(4)));  // (an array of the uint4 struct would be placed in scratch)
+typedef pv4 pv4_any __attribute__((aligned(2)));           // the same at any bf16 element
 
 struct PfGemmParams {
   const bf16_t* a;    // [M, K] row-major
@@ -181,7 +182,9 @@ __device__ __forceinline__ void store_tiles(const PfGemmParams& p, int row0, int
 //   2048 rows    64 -> 54.5     90 -> 49       205 -> 180     193 -> 103
 // LDS: A rows of 4 SUB 16-byte chunks, chunk c of row r at c ^ f(r), so that the 16 rows of a fragment
 // read hit different banks; W as its 1 KB tiles, those of one n-tile side by side.
-template <int BM, int BN, int WM, int WN, int SUB, int S, int EPI>
+// DIRECT false (operands that are not 16-byte aligned, which the direct loads need): a stage is loaded into registers
+// by ordinary loads and stored to its LDS slot one step later, behind that step's barrier.
+template <int BM, int BN, int WM, int WN, int SUB, int S, int EPI, bool DIRECT>
 __global__ void __launch_bounds__(64 * WM * WN, 1) prompt_gemm_kernel(PfGemmParams p) {
   constexpr int NW = WM * WN;
   constexpr int MB = BM / WM / 16, NB = BN / WN / 16;
@@ -191,6 +194,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 1) prompt_gemm_kernel(PfGemmPara
   constexpr int STAGE = (AI + WI) * 1024;
   static_assert(AI % NW == 0 && WI % NW == 0 && MB * WM * 16 == BM && NB * WN * 16 == BN, "tile split");
   static_assert(SUB == 2 || SUB == 4, "stages of 64 or 128 k");
+  static_assert(DIRECT || S >= 3, "a slot that is stored one step late is neither being read nor read next");
   static_assert(EPI != PEPI_SWIGLU || NB % 2 == 0, "gate / up pairs stay in one wavefront");
   __shared__ pv4 lds[S * STAGE / 16];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -238,10 +242,27 @@ __global__ void __launch_bounds__(64 * WM * WN, 1) prompt_gemm_kernel(PfGemmPara
       avoff[i] = (unsigned)min(row, last) * (unsigned)(p.K * 2) + (unsigned)((pc ^ (row & (C - 1))) * 16);
     }
   };
+  pv4 hold[DIRECT ? 1 : PER];   // the last requested stage (not DIRECT)
+  bool held = false;            // .. is still to be stored
   auto issue_one = [&](int i) __attribute__((always_inline)) {
-    const unsigned sb = lds0 + islot * STAGE;
-    if (i < PA) ring_load16(abase, avoff[i < PA ? i : 0], sb + (wave * PA + i) * 1024);
-    else ring_load16(wbase, wvoff[i < PA ? 0 : i - PA], sb + (AI + wave * PW + i - PA) * 1024);
+    if constexpr (DIRECT) {
+      const unsigned sb = lds0 + islot * STAGE;
+      if (i < PA) ring_load16(abase, avoff[i < PA ? i : 0], sb + (wave * PA + i) * 1024);
+      else ring_load16(wbase, wvoff[i < PA ? 0 : i - PA], sb + (AI + wave * PW + i - PA) * 1024);
+    } else {
+      hold[i] = *reinterpret_cast<const pv4_any*>(i < PA ? abase + avoff[i < PA ? i : 0] : wbase + wvoff[i < PA ? 0 : i - PA]);
+      held = true;
+    }
+  };
+  auto store_held = [&]() __attribute__((always_inline)) {   // into the slot before the cursor's
+    if constexpr (!DIRECT) {
+      if (held) {
+        pv4* st = lds + (islot == 0 ? S - 1 : islot - 1) * (STAGE / 16) + lane;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) st[(i < PA ? wave * PA + i : AI + wave * PW + i - PA) * 64] = hold[i];
+        held = false;
+      }
+    }
   };
   auto issue_next = [&]() __attribute__((always_inline)) {  // advance the issue cursor by one stage
     islot = islot + 1 == S ? 0 : islot + 1;
@@ -282,11 +303,14 @@ __global__ void __launch_bounds__(64 * WM * WN, 1) prompt_gemm_kernel(PfGemmPara
   auto step = [&](auto steady, const Frags& cur, Frags& nxt) __attribute__((always_inline)) {
     constexpr bool ST = decltype(steady)::value;
     const bool load = ST || g + S < G;
-    if constexpr (ST) ring_wait<PER * (S - 2)>();
-    else if (g + 1 < G) ring_wait_stages<PER, S - 2>(G - g - 2);
+    if constexpr (DIRECT) {
+      if constexpr (ST) ring_wait<PER * (S - 2)>();
+      else if (g + 1 < G) ring_wait_stages<PER, S - 2>(G - g - 2);
+    }
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
+    store_held();
     cslot = cslot + 1 == S ? 0 : cslot + 1;   // stage g + 1's slot
 #pragma unroll
     for (int gp = 0; gp < GP; ++gp) {
@@ -315,10 +339,11 @@ __global__ void __launch_bounds__(64 * WM * WN, 1) prompt_gemm_kernel(PfGemmPara
 #pragma unroll
       for (int i = 0; i < PER; ++i) issue_one(i);
       issue_next();
+      store_held();
     }
   }
   Frags f0, f1;
-  ring_wait_stages<PER, S - 1>(G - 1);
+  if constexpr (DIRECT) ring_wait_stages<PER, S - 1>(G - 1);
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < R; ++r) read_one(f0, 0, r);
@@ -558,14 +583,14 @@ __global__ void __launch_bounds__(256, 1) prompt_gemm_big_kernel(PfGemmParams p)
   }
 }
 
-template <int BM, int BN, int WM, int WN, int SUB, int S>
+template <int BM, int BN, int WM, int WN, int SUB, int S, bool DIRECT = true>
 int launch_tiles(PfGemmParams p, int epi, dim3 grid, hipStream_t stream) {
   p.mtiles = (p.M + BM - 1) / BM;
   p.ntiles = p.N / BN;
   constexpr int T = 64 * WM * WN;
-  if (epi == PEPI_STORE) prompt_gemm_kernel<BM, BN, WM, WN, SUB, S, PEPI_STORE><<<grid, T, 0, stream>>>(p);
-  else if (epi == PEPI_RES) prompt_gemm_kernel<BM, BN, WM, WN, SUB, S, PEPI_RES><<<grid, T, 0, stream>>>(p);
-  else prompt_gemm_kernel<BM, BN, WM, WN, SUB, S, PEPI_SWIGLU><<<grid, T, 0, stream>>>(p);
+  if (epi == PEPI_STORE) prompt_gemm_kernel<BM, BN, WM, WN, SUB, S, PEPI_STORE, DIRECT><<<grid, T, 0, stream>>>(p);
+  else if (epi == PEPI_RES) prompt_gemm_kernel<BM, BN, WM, WN, SUB, S, PEPI_RES, DIRECT><<<grid, T, 0, stream>>>(p);
+  else prompt_gemm_kernel<BM, BN, WM, WN, SUB, S, PEPI_SWIGLU, DIRECT><<<grid, T, 0, stream>>>(p);
   QWEN_RETURN_LAUNCH();
 }
 
@@ -613,6 +638,18 @@ extern "C" int qwen_gemm(const void* a, const void* w_tiled, void* out, int M, i
   p.out = (bf16_t*)out;
   p.M = M; p.N = N; p.K = K; p.ldo = ld_out;
   const int slots = std::max(1, device_cu_count() / 8);   // workgroups per XCD
+  // Direct loads want 16-byte aligned addresses; rows and tiles are multiples of 128 bytes, so the bases decide. All
+  // other operands are staged through registers, in the larger tile where the smaller one takes more than a round (us,
+  // smaller -> larger, N = 2688 and 2,048 rows: K = 2560 82 -> 53, K = 9728 311 -> 194). A load's latency shows in each
+  // k step: 29 us at 23 rows and K = 2560, 8.6 from aligned operands; at 16,384 rows and K = 9728 1,209, aligned 737.
+  if (((uintptr_t)a | (uintptr_t)w_tiled) & 15) {
+    const bool large = (long long)((M + 127) / 128) * (N / 64) > 8LL * slots;
+    const long long tiles = large ? (long long)((M + 255) / 256) * (N / 128) : (long long)((M + 127) / 128) * (N / 64);
+    if (tiles > 0x7fffff00LL) return QWEN_EARG;
+    const dim3 grid((unsigned)(8 * std::min<long long>((tiles + 7) / 8, slots)));
+    return large ? launch_tiles<256, 128, 4, 2, 2, 3, false>(p, epi, grid, stream)
+                 : launch_tiles<128, 64, 2, 2, 2, 6, false>(p, epi, grid, stream);
+  }
   int best = -1;
   long long least = 0, per_xcd = 0;
   for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); ++i) {
