@@ -91,8 +91,23 @@ def test_stream_is_the_choice_for_qwen_projections(qops):
     for M in (3, 20, 32):
         for N, K, pair, nt in ((6144, 2560, False, 2), (2560, 4096, False, 1), (19456, 2560, True, 6)):
             cfg = qops.gemm_config(M, N, K, pair)
-            assert isinstance(cfg, qops.StreamShape) and cfg == qops.stream_shape(M, nt)
-        assert len(qops.gemm_config(M, 2560, 9728)) == 3
+            assert isinstance(cfg, qops.StreamShape) and cfg.nt == nt
+        down = qops.gemm_config(M, 2560, 9728)
+        assert len(down) == 3 and not isinstance(down, qops.StreamShape)
+
+
+@pytest.mark.parametrize("M", [8, 20, 32])
+@pytest.mark.parametrize("kind,N,K", [("norm", 6144, 2560), ("res", 2560, 4096), ("silu", 19456, 2560)])
+def test_plain_copy_of_the_choice(qops, M, kind, N, K):
+    """A plain tuple with the values of the chosen shape is the general launch of the same projection, and
+    ``gemm_workspace_bytes`` of the chosen shape is enough for it."""
+    x, t, gain, res, want, bar = _case(qops, M, N, K, kind, seed=M + K)
+    cfg = qops.gemm_config(M, N, K, kind == "silu")
+    ws = qops.linear_workspace(qops.gemm_workspace_bytes(M, N, cfg), DEV)
+    for c in (cfg, tuple(cfg)):
+        got = qops.fused_linear(x, t, c, norm_w=gain if kind in ("norm", "silu") else None, eps=EPS,
+                                residual=res if kind == "res" else None, silu_pair=kind == "silu", workspace=ws)
+        assert bool(((got.float() - want).abs() <= bar).all()), (c, float(((got.float() - want).abs() - bar).max()))
 
 
 @pytest.mark.parametrize("kind,N,K,nt", [("plain", 64, 320, 1), ("res", 64, 256, 6), ("silu", 64, 256, 1),

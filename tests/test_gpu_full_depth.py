@@ -279,15 +279,20 @@ def test_b8_full_depth_hidden_states(full_gains, monkeypatch):
 
 
 def test_b32_full_depth_greedy_tokens(full_gains):
-    """c4's decode launch shapes (M = 32: skinny QKV / O / down with split-K, the rectangle gate/up,
-    the M = 32 LM head, one-split attention over 32 sequences) through 36 layers."""
+    """c4's decode launch shapes (M = 32: QKV, O and gate/up as weight streams of 2, 1 and 6 n-tiles per workgroup,
+    split-K down, the M = 32 LM head, one-split attention over 32 sequences) through 36 layers."""
+    from qwen_hip import ops
     eng, ref = full_gains
     B, Sp, Nn = 32, 64, 16
     prompt = _prompt(13, B, Sp)
     steps = list(eng.generate(prompt, Nn))
     assert len(steps) == Nn and all(len(s) == B for s in steps)
     b = eng.state.bufs[(0, 1)]
-    assert b.splits == 1 and not b.gemv and len(b.cfg["gu"]) == 4 and b.cfg["qkv"][2] > 1
+    assert b.splits == 1 and not b.gemv
+    names = {k: ops.gemm_kernel_name(b.M, c, k in ("qkv", "gu"), ops.EPI_STORE) for k, c in b.cfg.items()}
+    assert {k: n.split("<")[0] for k, n in names.items()} == {
+        "qkv": "decode_gemm_kernel", "o": "decode_gemm_kernel", "gu": "decode_gemm_kernel", "down": "skinny_gemm_kernel"}
+    assert [b.cfg[k].nt for k in ("qkv", "o", "gu")] == [2, 1, 6] and b.cfg["down"][2] > 1
     tokens = [[steps[n][i] for n in range(Nn)] for i in range(B)]
     check_tokens("c4 shapes B=32", ref, prompt, tokens)
 
