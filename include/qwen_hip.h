@@ -261,6 +261,10 @@ int qwen_spec_accept(const int64_t* nxt, const int64_t* tok, int64_t* hist, int3
 int qwen_gemm(const void* x, const void* w_tiled, void* out, int M, int N, int K, int ld_out, const void* residual,
               int epi, hipStream_t stream);
 
+/* Output tile of a qwen_gemm launch with aligned operands on `cus` CUs (0: the current device): rows << 16 | columns,
+ * 0 for sizes that it refuses. */
+int qwen_gemm_tile(int M, int N, int K, int cus);
+
 /* Causal attention of a prompt chunk: q [B, T, Nq, D] (normed + rotated queries of positions
  * p0 .. p0 + T - 1 of every sequence), caches [B, Nkv, CAP, D] already holding those
  * positions' keys / values; query t sees slots [0, p0 + t]. out [B, T, Nq * D] bf16.

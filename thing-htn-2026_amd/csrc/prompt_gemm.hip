@@ -607,20 +607,45 @@ int launch_big(PfGemmParams p, int epi, dim3 grid, hipStream_t stream) {
 // 64 k and `fixed` ns for filling the ring and the epilogue, [0] where one round leaves a quarter of the CUs idle (they
 // pull weights, and the others share less), [1] otherwise. Fitted on MI355X on the Qwen3-4B projections with cold
 // weights, every tile at 16 to 1,551 rows (the two largest also at 2,048 to 16,384). Rounds times that, the least
-// of it, picks the fastest or within 8 % of it.
+// of it, picks the fastest or within 8 % of it. `span`: n-tiles past its first whose weights a wavefront addresses by
+// 32-bit offsets from it.
 struct TileCost {
-  int bm, bn, sub;
+  int bm, bn, sub, span;
   int step[2], fixed[2];
 };
 constexpr TileCost TILES[] = {
-    {256, 256, 2, {1009, 1050}, {14600, 5500}}, {256, 128, 2, {585, 650}, {9400, 4300}},
-    {128, 128, 2, {410, 400}, {6400, 6000}},    {128, 64, 2, {271, 314}, {5900, 4400}},
-    {64, 128, 2, {285, 383}, {6400, 2100}},     {64, 64, 4, {172, 250}, {4500, 4200}},
-    {32, 128, 4, {250, 300}, {4300, 7400}},     {32, 64, 4, {129, 195}, {5000, 4500}},
-    {32, 32, 4, {96, 118}, {5400, 4400}},
+    {256, 256, 2, 15, {1009, 1050}, {14600, 5500}}, {256, 128, 2, 0, {585, 650}, {9400, 4300}},
+    {128, 128, 2, 0, {410, 400}, {6400, 6000}},     {128, 64, 2, 0, {271, 314}, {5900, 4400}},
+    {64, 128, 2, 0, {285, 383}, {6400, 2100}},      {64, 64, 4, 0, {172, 250}, {4500, 4200}},
+    {32, 128, 4, 1, {250, 300}, {4300, 7400}},      {32, 64, 4, 0, {129, 195}, {5000, 4500}},
+    {32, 32, 4, 0, {96, 118}, {5400, 4400}},
 };
 
+// The tile of a launch on slots x 8 CUs and the tiles per XCD's run; -1 where none fits.
+int choose_tile(int M, int N, int K, int slots, long long* per_xcd) {
+  int best = -1;
+  long long least = 0;
+  for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); ++i) {
+    const TileCost& t = TILES[i];
+    if (N % t.bn || K % (32 * t.sub)) continue;
+    if (((long long)t.span * (K / 32) + t.sub) * 1024 > 0xffffffffLL) continue;
+    const long long tiles = (long long)((M + t.bm - 1) / t.bm) * (N / t.bn), run = (tiles + 7) / 8;
+    if (tiles > 0x7fffff00LL) continue;
+    const int full = run * 4 > slots * 3;
+    const long long cost = (run + slots - 1) / slots * ((long long)(K / 64) * t.step[full] + t.fixed[full]);
+    if (best < 0 || cost < least) best = i, least = cost, *per_xcd = run;
+  }
+  return best;
+}
+
 }  // namespace
+
+extern "C" int qwen_gemm_tile(int M, int N, int K, int cus) {
+  if (M <= 0 || N <= 0 || K <= 0 || N % 128 || K % 64 || cus < 0 || (long long)M * K >= 0x7fffffffLL) return 0;
+  long long run = 0;
+  const int i = choose_tile(M, N, K, std::max(1, (cus ? cus : device_cu_count()) / 8), &run);
+  return i < 0 ? 0 : TILES[i].bm << 16 | TILES[i].bn;
+}
 
 extern "C" int qwen_gemm(const void* a, const void* w_tiled, void* out, int M, int N, int K, int ld_out,
                          const void* residual, int epi, hipStream_t stream) {
@@ -650,25 +675,14 @@ extern "C" int qwen_gemm(const void* a, const void* w_tiled, void* out, int M, i
     return large ? launch_tiles<256, 128, 4, 2, 2, 3, false>(p, epi, grid, stream)
                  : launch_tiles<128, 64, 2, 2, 2, 6, false>(p, epi, grid, stream);
   }
-  int best = -1;
-  long long least = 0, per_xcd = 0;
-  for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); ++i) {
-    const TileCost& t = TILES[i];
-    if (N % t.bn || K % (32 * t.sub)) continue;
-    // W offsets within a wavefront's part of a tile are 32 bits (none beyond one n-tile in the 128 x 64 and
-    // 32 x 32 tiles)
-    if (K >= 1 << 22 && !(t.bn == 64 && t.bm == 128) && t.bn != 32) continue;
-    const long long tiles = (long long)((M + t.bm - 1) / t.bm) * (N / t.bn), run = (tiles + 7) / 8;
-    if (tiles > 0x7fffff00LL) continue;
-    const int full = run * 4 > slots * 3;
-    const long long cost = (run + slots - 1) / slots * ((long long)(K / 64) * t.step[full] + t.fixed[full]);
-    if (best < 0 || cost < least) best = i, least = cost, per_xcd = run;
-  }
+  long long per_xcd = 0;
+  const int best = choose_tile(M, N, K, slots, &per_xcd);
   if (best < 0) return QWEN_EARG;
   // Persistent: at most one workgroup per CU. Idle CUs pull weights where they are a quarter or more (fewer fall behind
   // and only add traffic: down at 96 rows, 240 tiles of 32 x 32, 49 us with them, 22 without) and up to 1,024 rows
-  // (more do not wait for weights: down 77 -> 68 us at 1,000 rows, 75 -> 76 at 1,300, 97 -> 102 at 1,551).
-  p.pull = best > 0 && M <= 1024 && per_xcd * 4 <= slots * 3;
+  // (more do not wait for weights: down 77 -> 68 us at 1,000 rows, 75 -> 76 at 1,300, 97 -> 102 at 1,551). An n-tile's
+  // bytes are a 32-bit number there.
+  p.pull = best > 0 && M <= 1024 && per_xcd * 4 <= slots * 3 && K < 1 << 25;
   const dim3 grid((unsigned)(8 * (p.pull ? slots : std::min<long long>(per_xcd, slots))));
   switch (best) {
     case 0: return launch_big(p, epi, grid, stream);
