@@ -19,28 +19,13 @@
 // Chunks of more than 16 tokens take pf_attn_wide_kernel (16 or 32 query tokens per 4-wavefront workgroup, two
 // workgroups per CU), described at its definition below.
 #include "common.h"
+#include "lds_ring.h"
 
 namespace {
 
 // 16 bytes held as a native vector: arrays of these stay in VGPRs (an array of the HIP uint4
 // struct is placed in scratch memory, and every load into it then waits at its store).
 typedef unsigned pv4 __attribute__((ext_vector_type(4)));
-
-// Direct global -> LDS load of 16 bytes per lane, from a wavefront-uniform base in SGPRs and a
-// 32-bit per-lane byte offset (no 64-bit address arithmetic per load): lane l's bytes land at
-// LDS byte address `lds_addr` + 16 l (lds_addr wavefront-uniform, held in M0). Written as inline
-// assembly so that the compiler does not treat it as an LDS store: it would otherwise make every
-// later LDS read wait for all such loads. The caller therefore waits for them itself
-// (lds_dma_wait) before the barrier after which they are read; waits the compiler places for its
-// own loads stay correct, only more conservative (loads complete in issue order). s_nop covers
-// the M0 write -> LDS-DMA hazard.
-__device__ __forceinline__ void lds_dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-__device__ __forceinline__ void lds_dma16_so(const void* sbase, unsigned voff, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :
-               : "v"(voff), "s"(sbase), "s"(lds_addr)
-               : "memory", "m0");
-}
 
 // ------------------------------------------------------------------ causal flash attention
 constexpr int AD = 128;      // head dim
@@ -342,14 +327,14 @@ __global__ void __launch_bounds__(AW2 * 64, 2) pf_attn_wide_kernel(PfAttnParams 
     const unsigned lds0 = (k ? lds_k : lds_v) + (unsigned)((buf * AKB + 4 * AGPW * wave) * 256);
     if ((blk + 1) * AKB <= kmax) {
 #pragma unroll
-      for (int i = 0; i < AGPW; ++i) lds_dma16_so(sb, k ? koff[i] : voff[i], lds0 + i * 1024);
+      for (int i = 0; i < AGPW; ++i) ring_load16(sb, k ? koff[i] : voff[i], lds0 + i * 1024);
     } else {
       const int last = kmax - 1 - blk * AKB;   // last row of the block below kmax (>= 0)
 #pragma unroll
       for (int i = 0; i < AGPW; ++i) {
         const int r = 4 * (AGPW * wave + i) + srow;   // row of the block
         const unsigned off = k ? koff[i] : voff[i];
-        lds_dma16_so(sb, r <= last ? off : off - (unsigned)((r - last) * 256), lds0 + i * 1024);
+        ring_load16(sb, r <= last ? off : off - (unsigned)((r - last) * 256), lds0 + i * 1024);
       }
     }
   };
@@ -366,7 +351,7 @@ __global__ void __launch_bounds__(AW2 * 64, 2) pf_attn_wide_kernel(PfAttnParams 
 
   issue_kv(0, 0, true);
   issue_kv(0, 0, false);
-  lds_dma_wait();
+  ring_wait<0>();
   __syncthreads();
   for (int blk = 0; blk < nblk; ++blk) {
     const int buf = blk & 1;
@@ -459,7 +444,7 @@ __global__ void __launch_bounds__(AW2 * 64, 2) pf_attn_wide_kernel(PfAttnParams 
           o[mt][nd] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vv), as_bf16x8(pb[mt][kk]), o[mt][nd], 0, 0, 0);
       }
     }
-    lds_dma_wait();  // this wavefront's next-block loads have landed ...
+    ring_wait<0>();  // this wavefront's next-block loads have landed ...
     __syncthreads();  // ... and, past the barrier, every wavefront's
   }
 
