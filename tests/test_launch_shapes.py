@@ -1,6 +1,7 @@
 """Launch shapes of the decode projections (``qwen_hip.ops``): host arithmetic only."""
 
 import copy
+import json
 import os
 import pickle
 
@@ -51,3 +52,26 @@ def test_workspace_of_every_form():
             assert ops.gemm_workspace_bytes(M, N, cfg) == ops.gemm_workspace_bytes(M, N, tuple(cfg))
     assert ops.gemm_workspace_bytes(32, 6144, ops.gemm_config(32, *QKV)) > 0
     assert ops.gemm_workspace_bytes(32, 6144, (2,)) == 0
+
+
+def test_measured_traffic_is_of_the_launches_that_run():
+    """``bench.py`` looks measured HBM bytes up by the kernel's name: the committed names are those that the
+    MFMA projections launch now (M = sequences x tokens per step; the other entries are GEMVs and attention)."""
+    import bench
+    with open(bench.TRAFFIC_FILE) as f:
+        traffic = json.load(f)
+    roles = {"gu": (GU, True, ops.EPI_SWIGLU), "o": (O, False, ops.EPI_RES), "qkv": (QKV, True, ops.EPI_STORE),
+             "down": (DOWN, False, ops.EPI_RES)}
+    rows = {"c3": 8, "c4": 32, "c5": 4 * bench.SPEC_T}
+    seen = 0
+    for key, entry in traffic.items():
+        config, _, role = key.partition("_")
+        if config not in rows or key == "c4":   # (c4's own entry is the attention's)
+            continue
+        shape, norm, epi = roles[role or "gu"]
+        M = rows[config]
+        name = ops.gemm_kernel_name(M, ops.gemm_config(M, *shape), norm, epi)
+        assert entry["kernel"] == name, key
+        assert bench.measured_traffic(key, name) == entry["bytes_per_launch"]
+        seen += 1
+    assert seen == 6
