@@ -2,13 +2,13 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--config default|c2|c3|c4|c5]
 
-BASELINE.json's metric is "decode tok/s at B=1 and B=32 (Qwen3-4B bf16); HBM GB/s as % of peak".
+The metric is "decode tok/s at B=1 and B=32 (Qwen3-4B bf16); HBM GB/s as % of peak".
 The default run measures both halves in one invocation on random-init Qwen3-4B bf16 weights
 (seed 0), greedy decoding through the engine's own ``generate()``:
 
-* ``value`` (B = 1, configs[1] "c2": a 128-token uniform-random prompt, 256 decode steps);
-* ``b32`` (B = 32, configs[3] "c4": 8192-token prompts, 256 decode steps, ~37 GiB of KV cache);
-* ``c3`` (B = 8, configs[2]) and ``c5`` (the speculative verify step, configs[4]) as further
+* ``value`` (B = 1, "c2": a 128-token uniform-random prompt, 256 decode steps);
+* ``b32`` (B = 32, "c4": 8192-token prompts, 256 decode steps, ~37 GiB of KV cache);
+* ``c3`` (B = 8) and ``c5`` (the speculative verify step) as further
   blocks of the same line, so that every decode config is timed in the default run.
 
 Each is timed as follows. The batch state is built, certified and its step graph recorded
@@ -56,7 +56,7 @@ sys.path.insert(0, ROOT)
 HBM_PEAK = 8.0e12        # MI355X HBM3E, bytes/s
 MFMA_BF16_PEAK = 2.5e15  # MI355X dense bf16 matrix peak, flop/s
 CONFIGS = {
-    # name: (B, prompt length, decode steps), BASELINE.json configs[1..4]
+    # name: (B, prompt length, decode steps)
     "c2": (1, 128, 256),
     "c3": (8, 2048, 512),
     "c4": (32, 8192, 256),

@@ -2,7 +2,7 @@
 
 TEST INFRASTRUCTURE ONLY. Nothing in the product (``thing-htn-2026_amd/``)
 imports, links or runs anything from this package. It is used by ``tests/``
-as the checker, by ``__graft_entry__.smoke()`` to check one small GPU call,
+as the oracle, by ``__graft_entry__.smoke()`` to check one small GPU call,
 and by ``bench.py``'s ``cpu_baseline`` leg as the timed CPU restatement.
 
 Modules

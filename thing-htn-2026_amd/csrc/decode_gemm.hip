@@ -17,8 +17,9 @@
 //   QKV       8.4 -> 8.3       8.8 -> 8.5       9.8 -> 9.0       11.8 -> 10.1     13.5 -> 10.7
 //   O         7.3 -> 6.4       7.4 -> 7.1       8.7 -> 7.8       10.2 -> 8.7      11.2 -> 9.5
 //   gate/up   20.6 -> 20.0     20.5 -> 19.4     23.5 -> 19.7     25.0 -> 20.9     25.1 -> 21.1
-// The down projection (k = 9728, 160 workgroups) stays with gemm.hip's split of k: its activations are 2 M / 16 times
-// the bytes of a 16-column workgroup's weights, and it measured 13.4 -> 14.9 us at M = 8, 17.1 -> 18.6 at 32.
+// The down projection (k = 9728) stays with gemm.hip's split of k in three, 240 workgroups: here 160 would each move
+// its 311 KB of weights and M / 16 times that of activations, while 96 CUs idle. 12.1 -> 12.5 us at M = 8, 12.4 -> 14.7
+// at 16, 16.5 -> 18.6 at 32 (and 12.0 -> 11.3 at 3).
 #include "common.h"
 #include "lds_ring.h"
 

@@ -174,12 +174,12 @@ __device__ __forceinline__ void store_tiles(const PfGemmParams& p, int row0, int
 // the multiplications of this stage between the next one's LDS reads and the loads of the stage S on,
 // into the slot just left. What bounds it at few rows is the loads, see pull_weights (a wavefront that runs ahead in
 // the same CU made every shape 5 - 40 % slower, non-temporal W loads 10 - 50 %). Against the one 256 x 256
-// tile that all shapes ran before (Qwen3-4B, cold weights, us per launch):
+// tile that all shapes ran before (Qwen3-4B, us per launch, graph replays over 1.2 GB of weights):
 //                QKV            O              gate/up        down
-//   23 rows      50 -> 10.5     77 -> 10.8     65 -> 21.6     176 -> 21
-//   128 rows     53 -> 13.4     84 -> 12.5     73 -> 27       185 -> 25
-//   512 rows     58 -> 23.2     89 -> 23.4     78 -> 61       191 -> 48
-//   2048 rows    64 -> 54.5     90 -> 49       205 -> 180     193 -> 103
+//   23 rows      57 -> 10.7     89 -> 11.0     62 -> 23.0     206 -> 20.6
+//   128 rows     63 -> 13.6     97 -> 12.7     70 -> 29.4     220 -> 25.3
+//   512 rows     72 -> 24.4     105 -> 23.2    75 -> 63       237 -> 48
+//   2048 rows    69 -> 58       103 -> 51      207 -> 187     223 -> 109
 // LDS: A rows of 4 SUB 16-byte chunks, chunk c of row r at c ^ f(r), so that the 16 rows of a fragment
 // read hit different banks; W as its 1 KB tiles, those of one n-tile side by side.
 // DIRECT false (operands that are not 16-byte aligned, which the direct loads need): a stage is loaded into registers
@@ -374,10 +374,11 @@ __global__ void __launch_bounds__(64 * WM * WN, 1) prompt_gemm_kernel(PfGemmPara
 // (16,384 rows): reads and loads in one group before 8 MFMAs and the cursors after the phase 1,280 TFLOP/s,
 // interleaved 1,315, cursors in between as well 1,390 (gate/up). A load is requested two phases before
 // the barrier that waits for it (vmcnt(16): the last two phases' loads stay in flight).
-// Against the 8-wavefront kernel with two full stages that it replaces, per launch at 16,384 rows: QKV 416 -> 350 us
-// (1,473 TFLOP/s), O 315 -> 273, gate/up + SwiGLU 1,333 -> 1,176 (1,388), down 742 -> 599 (1,362). 64 MFMAs alone on
-// every SIMD, random operands in registers, run at 1,766 TFLOP/s (the chip lowers its clock), with this phase's
-// LDS reads, barrier and L2-resident loads at 1,531.
+// Against the 8-wavefront kernel with two full stages that it replaces, us per launch at 16,384 rows, the same launch
+// back to back: QKV 425 -> 370, O 322 -> 283, gate/up + SwiGLU 1,363 -> 1,221, down 750 -> 633; between the other kernels
+// of a prompt forward 352 / 284 / 1,179 / 604 (1,464 / 1,210 / 1,385 / 1,352 TFLOP/s; O and down are 2.5 rounds
+// of tiles that cost three). 64 MFMAs alone on every SIMD, random operands in registers, run at 1,766 TFLOP/s (the chip
+// lowers its clock), with this phase's LDS reads, barrier and L2-resident loads at 1,531.
 constexpr int GM = 256, GN = 256;
 constexpr int G_ASLOTS = 3, G_WSLOTS = 4;
 constexpr int G_ABYTES = 32 * 1024;   // 256 A rows x 64 k; 16-byte chunk c of row r at c ^ (r % 8)
