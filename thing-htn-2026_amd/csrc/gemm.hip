@@ -180,8 +180,9 @@ struct AOperand {
 // issues are unconditional (a conditional issue makes the compiler's wait at the
 // join count the batch just requested, which serialises the pipeline) and the
 // last one or two batches form a separate tail. Within a batch, weight slots
-// past k1 read a cache-resident dummy (the activation rows) and the activation
-// slots re-read step k1-1; both meet a zero A operand. With `stats_after_first`
+// past k1 re-read the wavefront's first weight tile and the activation slots
+// step k1-1; both meet a zero A operand (not the activation rows in place of
+// weights: zero times one that is not finite would reach every row). With `stats_after_first`
 // the A operand's RMSNorm statistics are requested before the first weights and
 // added once those are in flight.
 template <int MT, int NTW, int U, bool NORM, typename AfterFirst>
@@ -197,7 +198,7 @@ __device__ __forceinline__ void accumulate(const GemmParams& p, AOperand<MT, NOR
   struct Batch {
     uint4 bt[U][NTW], at[U][MT], gt[U];
   };
-  const uint4* dummy = reinterpret_cast<const uint4*>(p.x) + lane;
+  const uint4* dummy = wt + wrow[0] + (size_t)k0 * 64;
   auto issue = [&](Batch& b, int kt) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
