@@ -116,3 +116,21 @@ def test_stream_rejects_unfit_shapes(qops, kind, N, K, nt):
     x, t, gain, res, _, _ = _case(qops, 4, N, K, "silu" if kind == "silu" else "plain", seed=1)
     with pytest.raises(RuntimeError):
         _run(qops, x, t, gain, res, kind, nt)
+
+
+@pytest.mark.parametrize("off", [1, 2, 4, 7])
+@pytest.mark.parametrize("kind,N,K,nt", [("norm", 512, 1280, 2), ("res", 256, 512, 1), ("silu", 384, 256, 6)])
+@pytest.mark.parametrize("M", [3, 20])
+def test_stream_operands_off_a_16_byte_boundary(qops, M, kind, N, K, nt, off):
+    """Rows and weights that start at any bf16 element: the stream hands these on, the result is held to the same bar."""
+    x, t, gain, res, want, bar = _case(qops, M, N, K, kind, seed=M + off)
+
+    def shifted(v):
+        flat = torch.empty(v.numel() + off, dtype=BF16, device=DEV)[off:]
+        assert flat.data_ptr() % 16 == 2 * off
+        return flat.view(v.shape).copy_(v)
+
+    ts = qops.TiledWeight(shifted(t.data), N, K, t.pair)
+    for xx, tt in ((shifted(x), t), (x, ts), (shifted(x), ts)):
+        got, _ = _run(qops, xx, tt, gain, res, kind, nt)
+        assert bool(((got.float() - want).abs() <= bar).all()), float(((got.float() - want).abs() - bar).max())
